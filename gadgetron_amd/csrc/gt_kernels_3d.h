@@ -331,16 +331,17 @@ __global__ __launch_bounds__(64, 3) void nc2c_mfma3d_kernel(
 #pragma unroll
     for (int u = 0; u < kDV; u++) dv[u] = 1.0f;
 
-    // entries [cb, cb + 32) of [begin, end), end > begin; lanes past end load a
-    // valid address, and stage gives those entries zero weights (a select here
-    // would wait for the loads just issued)
+    // entries [cb, cb + 32) of [begin, end), end > begin; lanes past end load the
+    // last entry's words (its sample and rows: the padding reads no other sample, and
+    // brings nothing of its own to the scale R), and stage gives those entries zero
+    // weights (a select here would wait for the loads just issued)
     auto load = [&](uint32_t cb) {
         const uint32_t cv = min(cb, it.end - 1), n = min(it.end - cv, (uint32_t)k3MK);
         const float4* w4 = reinterpret_cast<const float4*>(wt) + (size_t)cv * kF4;
         const uint32_t last = n * kF4 - 1;
 #pragma unroll
         for (int t = 0; t < 3; t++) wreg[t] = w4[min((uint32_t)(lane + kLanes * t), last)];
-        hreg = (hd + (size_t)cv * 2)[min((uint32_t)lane, 2 * n - 1)];
+        hreg = (hd + (size_t)cv * 2)[head_word((uint32_t)lane, n)];
     };
     // entries from cb, as loaded, to chunk buffer b
     auto stage = [&](uint32_t cb, int b) {

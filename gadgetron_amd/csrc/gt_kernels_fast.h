@@ -13,6 +13,7 @@
 // caller's [x, y, batch] layout of convolve().
 #pragma once
 
+#include "gt_index.h"
 #include "gt_kernels.h"
 
 namespace gt {

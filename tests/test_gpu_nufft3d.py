@@ -207,6 +207,64 @@ def test_3d_nc2c_chunk_remainders(gpu, M, C, dcw):
     assert rel_l2(outs[0], outs[1]) <= TOL
 
 
+class Prefix:
+    """The first elements of a larger device array, as an array of their own."""
+
+    def __init__(self, whole, shape):
+        self.whole, self.shape = whole, shape
+
+    def data_ptr(self):
+        return self.whole.data_ptr()
+
+
+@pytest.mark.parametrize("C", [3, 8, 11])
+@pytest.mark.parametrize("M", [1, 31, 33, 200])
+def test_3d_nc2c_reads_its_own_samples(gpu, M, C):
+    # NaN right behind the samples and the weights of a plan of few samples: none of it
+    # is read, so the grid is the same as without
+    say(f"3D 32^3, {M} samples, {C} coils, NaN behind samples and weights")
+    rng = np.random.default_rng(M + C)
+    plan = NFFTPlan([32, 32, 32], None, W=5.5, os_factor=1.5)
+    plan.preprocess(dev((rng.uniform(0.0, 0.02, (1, M, 3)) + 0.1).astype(np.float32)))
+    smp = tj.complex_normal(rng, (C, 1, M))
+    w = rng.uniform(0.1, 1.0, (C, 1, M)).astype(np.float32)
+    outs = []
+    for pad in (0.0, np.nan):
+        s = dev(np.concatenate([smp.reshape(-1), np.full(1024, pad, np.complex64)]), np.complex64)
+        d = dev(np.concatenate([w.reshape(-1), np.full(1024, pad, np.float32)]), np.float32)
+        out = DeviceArray.zeros((C, 1, 32, 32, 32), np.complex64)
+        plan.compute(Prefix(s, smp.shape), out, Prefix(d, w.shape), CM.BACKWARDS_NC2C)
+        plan.synchronize()
+        outs.append(out.numpy())
+    assert np.all(np.isfinite(outs[1]))
+    assert np.array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("bad", [0, 1, 128, 255])
+def test_3d_nc2c_bad_sample_stays_in_its_tiles(gpu, bad):
+    # one NaN sample: the 8 x 8 x 4 tiles that its window does not touch are as without
+    # it (bitwise: neither their sums nor their scales see it)
+    say(f"3D 32^3, 600 samples, 8 coils, sample {bad} is NaN")
+    rng = np.random.default_rng(bad)
+    M, C, G = 600, 8, 48
+    traj = rng.uniform(-0.5, 0.5, (1, M, 3)).astype(np.float32)
+    plan = NFFTPlan([32, 32, 32], None, W=5.5, os_factor=1.5)
+    plan.preprocess(dev(traj))
+    smp = tj.complex_normal(rng, (C, 1, M))
+    with_nan = smp.copy()
+    with_nan[:, 0, bad] = np.nan
+    a = conv(plan, smp, (C, 1, G, G, G), NFFT_conv_mode.NC2C)
+    b = conv(plan, with_nan, (C, 1, G, G, G), NFFT_conv_mode.NC2C)
+    touched = np.ones((G, G, G), bool)
+    for d, T in enumerate((8, 8, 4)):  # x, y, z
+        p = (traj[0, bad, d] + np.float32(0.5)) * np.float32(G)
+        cells = np.arange(int(np.ceil(p - 2.75)), int(np.floor(p + 2.75)) + 1) % G
+        line = np.isin(np.arange(G) // T, cells // T)
+        touched &= line.reshape([-1 if i == 2 - d else 1 for i in range(3)])
+    assert touched.any() and not touched.all()
+    assert np.array_equal(a[:, 0, ~touched], b[:, 0, ~touched])
+
+
 def test_3d_convolve_accumulate(gpu):
     say("3D 32^3, 3 coils: convolve with accumulate, both directions")
     N = [32, 32, 32]
