@@ -263,8 +263,11 @@ __global__ __launch_bounds__(64, 3) void nc2c_reg3d_kernel(
 // entries k of s[q][k] w[k][cell], w[k][cell] = wx_k[x] wy_k[y] wz_k[z]: each
 // chunk of 32 table entries is one K = 32 step of v_mfma_f32_16x16x32_f16 on
 // 16 blocks of 16 cells (block = plane z and rows 2p, 2p + 1), with the
-// split-fp16 products hi*hi + hi*lo + lo*hi and the power-of-two scales of
-// nc2c_mfma2d_kernel (relative error about 2^-22 per product, FP32 sums).  The
+// split-fp16 products hi*hi + hi*lo + lo*hi of nc2c_mfma2d_kernel and power-of-two
+// scales, one of the weights and one of each row of samples, so that a coil's accuracy
+// does not depend on the others' (relative error against double sums over the same
+// weights, white data, any ratio of coils: 8.7e-8; with one scale for the tile's
+// samples and weights of at most 1, 2.1e-7, and 5e-4 for a coil 1e-7 of the largest).  The
 // plane weights go with the samples: A_z = s wz (4 planes), B_p = wx wy (4 row
 // pairs), so 8 products are formed and split per chunk for the 16 blocks.  The
 // vector operations of the split bound it: 16 products of s with (wx wy wz),
@@ -280,6 +283,7 @@ __global__ __launch_bounds__(64, 3) void nc2c_reg3d_kernel(
 // t, B column l % 16 at the same k; accumulator register r of lane l is row
 // 4 (l / 16) + r, column l % 16.
 // ---------------------------------------------------------------------------
+constexpr float k3WeightTop = 16384.0f;  // the largest wx wy: those of a window's edge keep a normal low half
 constexpr int k3MK = 32;         // table entries per chunk (the MFMA's K)
 constexpr int k3MS = k3MK + 4;   // floats per LDS row of entry-contiguous data
 struct Mf3Lds {
@@ -319,7 +323,7 @@ __global__ __launch_bounds__(64, 3) void nc2c_mfma3d_kernel(
     mf_float4 acc[16];  // block = z * 4 + p
 #pragma unroll
     for (int b = 0; b < 16; b++) acc[b] = mf_float4{0.0f, 0.0f, 0.0f, 0.0f};
-    float R = 0.0f;  // sample scale (0: not set yet)
+    float R = 0.0f;  // scale of the samples of row `row` (0: not set yet)
 
     constexpr int kDV = DM == 2 ? 4 : 1;
     float4 wreg[3];
@@ -408,22 +412,25 @@ __global__ __launch_bounds__(64, 3) void nc2c_mfma3d_kernel(
         const float4* xa = reinterpret_cast<const float4*>(xs + row * k3MS + 8 * kh);
         const float4 a0 = xa[0], a1 = xa[1];
         mf_float8 x = mf_float8{a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w} * Rt;
-        const float m = mf_absmax(x);
-        if (__builtin_amdgcn_ballot_w64(m > (R == 0.0f ? 0.0f : 32768.0f))) {
-            const float mx = mf_wave_max(m);  // of x = samples * Rt
-            int e;
-            frexpf(mx, &e);                   // mx < 2^e
-            e = min(max(e, -100), 140);       // keep R and 1 / R finite
-            const float fs = ldexpf(1.0f, 12 - e);
-            if (R != 0.0f) {
+        const float m = mf_absmax(x), top = R == 0.0f ? 0.0f : 32768.0f;
+        if (__builtin_amdgcn_ballot_w64(m > top)) {
+            // of x = samples * Rt, over the four lanes of the row
+            float mx = fmaxf(m, __shfl_xor(m, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const bool on = mx > top;
+            const int e = max((int)(__float_as_uint(mx) >> 23) - 126, -100);  // mx < 2^e; R and 1 / R stay finite
+            const float fs = on ? ldexpf(1.0f, 12 - e) : 1.0f;
 #pragma unroll
-                for (int bl = 0; bl < 16; bl++) acc[bl] *= fs;  // powers of two: exact
+            for (int r = 0; r < 4; r++) {
+                const float f = __shfl(fs, 4 * kh + r);  // of the accumulators' rows
+#pragma unroll
+                for (int bl = 0; bl < 16; bl++) acc[bl][r] *= f;  // powers of two: exact
             }
             x *= fs;
-            R = Rt * fs;
+            if (on) R = Rt * fs;
         }
         // A of each plane: samples times the plane's weights (sz and sxy are powers of
-        // two that bring the largest wz and wx wy to at most 1)
+        // two that bring the largest wz to at most 1, the largest wx wy to k3WeightTop)
         x *= sz;
         mf_half8 xh[k3T2], xl[k3T2];
 #pragma unroll
@@ -474,7 +481,7 @@ __global__ __launch_bounds__(64, 3) void nc2c_mfma3d_kernel(
 
     // write-out through LDS one plane at a time: xp[q][y * 8 + x], then lanes
     // run along (re/im, x) for coalesced stores of (coil, y) rows
-    const float outs = R > 0.0f ? 1.0f / (R * sxy * sz) : 0.0f;  // powers of two: exact
+    const float out = R > 0.0f ? 1.0f / (R * sxy * sz) : 0.0f;  // of row `row`; powers of two: exact
     const int f = (int)(it.key / (uint32_t)g.ntiles_total);
     int org[3];
     tile_origin3((int)(it.key % (uint32_t)g.ntiles_total), g, org);
@@ -485,7 +492,7 @@ __global__ __launch_bounds__(64, 3) void nc2c_mfma3d_kernel(
         for (int pp = 0; pp < 4; pp++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
-                xp[(4 * kh + r) * kOut + (2 * pp + cyo) * k3T0 + cx] = acc[z * 4 + pp][r] * outs;
+                xp[(4 * kh + r) * kOut + (2 * pp + cyo) * k3T0 + cx] = acc[z * 4 + pp][r] * __shfl(out, 4 * kh + r);
         __syncthreads();
         const int gz = org[2] + z;
 #pragma unroll 4
