@@ -85,3 +85,47 @@ def errors(D, N, W, C, M, mode, unequal):
 @pytest.mark.parametrize("C", [1, 3, 8])
 def test_3d_nc2c(C, unequal):
     assert max(errors(3, 32, 5.5, C, 3000, NFFT_conv_mode.NC2C, unequal)) <= SPLIT
+
+
+@pytest.mark.parametrize("unequal", [False, True])
+@pytest.mark.parametrize("C", [1, 3, 8])
+@pytest.mark.parametrize("W", [3.0, 5.5, 6.5])
+def test_2d_nc2c_few_coils(W, C, unequal):
+    assert max(errors(2, 64, W, C, 4000, NFFT_conv_mode.NC2C, unequal)) <= FP32
+
+
+def test_2d_nc2c_few_coils_dense():
+    # 2900 entries a tile: items of 512, 110 terms a cell in each, in chains of at most
+    # 4 of 16 entries, pairs of those and 16 pairs: 2.4e-8 sqrt(2 + 2 + 1 + 8) = 8.7e-8
+    assert max(errors(2, 32, 5.5, 8, 40000, NFFT_conv_mode.NC2C, True)) <= 1.3 * FP32
+
+
+@pytest.mark.parametrize("M", [300, 9000])  # one chunk a tile; several, and split tiles
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_2d_nc2c_bad_sample_stays_in_its_window(M, bad):
+    # cells whose window does not hold the sample, and other coils, are as without it
+    print(f"2D 64^2, {M} samples, 8 coils, one sample {bad}", flush=True)
+    rng = np.random.default_rng(M)
+    nos, C, W, j = 96, 8, 5.5, 17
+    k = rng.uniform(-0.5, 0.5, (1, M, 2)).astype(np.float32)
+    k[0, : M // 2] *= 0.1
+    plan = NFFTPlan([64, 64], None, W=W, os_factor=1.5)
+    plan.preprocess(DeviceArray.from_numpy(k))
+    x = (rng.standard_normal((C, 1, M)) + 1j * rng.standard_normal((C, 1, M))).astype(np.complex64)
+    y = x.copy()
+    y[3, 0, j] = bad
+    outs = []
+    for s in (x, y):
+        out = DeviceArray.zeros((C, 1, nos, nos), np.complex64)
+        plan.convolve(DeviceArray.from_numpy(s), out, NFFT_conv_mode.NC2C)
+        outs.append(out.numpy()[:, 0])
+    a, b = outs
+    hit = np.zeros((nos, nos), bool)
+    win = [np.arange(np.ceil(p - W / 2), np.floor(p + W / 2) + 1).astype(int) % nos
+           for p in (k[0, j] + np.float32(0.5)) * np.float32(nos)]
+    hit[np.ix_(win[1], win[0])] = True
+    assert np.array_equal(np.delete(a, 3, 0), np.delete(b, 3, 0))
+    assert not np.isfinite(b[3][hit]).any()
+    assert np.isfinite(b[3][~hit]).all()
+    # those of the same tiles are summed again, in another order
+    assert np.linalg.norm(b[3][~hit] - a[3][~hit]) <= 2 * FP32 * np.linalg.norm(a[3])
