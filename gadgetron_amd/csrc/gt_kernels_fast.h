@@ -132,12 +132,15 @@ __global__ void c2nc_table2d_kernel(const float* __restrict__ p, const uint32_t*
 // Weight rows of the matrix-core C2NC, 32 floats per entry: the sample's x
 // weights at the 16 staged columns, then its y weights at the 16 staged rows
 // (staged coordinates start at tile origin - floor(r); zero outside the
-// window), each axis scaled by a power of two (sx, sy) so no weight exceeds 1.
+// window), each axis scaled by a power of two (sx, sy).  The last float, past the
+// staged rows, holds the first column + 16 first row (as an integer) of KW columns
+// and rows inside the staged ones that hold the window.
 template <int KW>
 __device__ __forceinline__ void c2nc_wtable2d_entry(long long e, const float* __restrict__ p,
                                                     const uint32_t* __restrict__ list, const GridGeom& g, float sx,
                                                     float sy, float* __restrict__ wtab) {
-    static_assert(c2nc_extent(8, KW) <= 16, "a staged row holds 16 cells");
+    constexpr int E = c2nc_extent(8, KW);
+    static_assert(E < 16, "fewer staged rows than the 16 weights");
     const uint32_t j = list[e];
     const int fr = (int)floorf(g.radius);
     float wx[KW], wy[KW];
@@ -163,6 +166,7 @@ __device__ __forceinline__ void c2nc_wtable2d_entry(long long e, const float* __
             if (c == by + i) ry[c] = wy[i] * sy;
         }
     }
+    ry[15] = __uint_as_float((uint32_t)(min(bx, 16 - KW) + 16 * min(by, E - KW)));
     float4* t = reinterpret_cast<float4*>(wtab + e * 32);
 #pragma unroll
     for (int q = 0; q < 4; q++) {

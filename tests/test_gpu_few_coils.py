@@ -1,6 +1,5 @@
-"""2D gridding of 1 to 16 coils on the matrix cores (8-coil NC2C waves, C2NC
-workgroups of 1, 2, 4, 8 and 16 coils): every coil count at which the launch
-changes or leaves lanes idle, every kernel width with its own staging, several
+"""2D gridding of 1 to 16 coils (NC2C waves of 8 coils, C2NC workgroups of 1, 2, 4
+and 8): every coil count at which the launch changes or leaves lanes idle, every kernel width with its own staging, several
 frames, samples per tile from none to several blocks and split tiles, each kind of
 dcw, and accumulation.
 

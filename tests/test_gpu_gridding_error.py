@@ -129,3 +129,36 @@ def test_2d_nc2c_bad_sample_stays_in_its_window(M, bad):
     assert np.isfinite(b[3][~hit]).all()
     # those of the same tiles are summed again, in another order
     assert np.linalg.norm(b[3][~hit] - a[3][~hit]) <= 2 * FP32 * np.linalg.norm(a[3])
+
+
+@pytest.mark.parametrize("unequal", [False, True])
+@pytest.mark.parametrize("C", [1, 2, 4, 8, 16])
+@pytest.mark.parametrize("W", [3.0, 5.5, 6.5])
+def test_2d_c2nc_few_coils(W, C, unequal):
+    assert max(errors(2, 64, W, C, 4000, NFFT_conv_mode.C2NC, unequal)) <= FP32
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_2d_c2nc_bad_cell_stays_in_its_windows(bad):
+    # samples whose window's slots do not reach the cell, and other coils, are as without it
+    print(f"2D 64^2, 8 coils, one grid cell {bad}", flush=True)
+    rng = np.random.default_rng(2)
+    nos, C, W, M = 96, 8, 5.5, 5000
+    k = rng.uniform(-0.5, 0.5, (1, M, 2)).astype(np.float32)
+    plan = NFFTPlan([64, 64], None, W=W, os_factor=1.5)
+    plan.preprocess(DeviceArray.from_numpy(k))
+    x = (rng.standard_normal((C, 1, nos, nos)) + 1j * rng.standard_normal((C, 1, nos, nos))).astype(np.complex64)
+    y = x.copy()
+    y[3, 0, 40, 51] = bad
+    outs = []
+    for g in (x, y):
+        out = DeviceArray.zeros((C, 1, M), np.complex64)
+        plan.convolve(DeviceArray.from_numpy(g), out, NFFT_conv_mode.C2NC)
+        outs.append(out.numpy()[:, 0])
+    a, b = outs
+    p = (k[0] + np.float32(0.5)) * np.float32(nos)
+    d = np.abs((p - np.array([51, 40], np.float32) + nos / 2) % nos - nos / 2)
+    inside, near = (d <= W / 2).all(axis=1), (d <= W / 2 + 1).all(axis=1)  # a slot of weight 0 lies next to the window
+    assert inside.any() and not np.isfinite(b[3][inside]).any()
+    assert np.array_equal(a[3][~near], b[3][~near])
+    assert np.array_equal(np.delete(a, 3, 0), np.delete(b, 3, 0))
