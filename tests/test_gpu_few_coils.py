@@ -1,7 +1,7 @@
 """2D gridding of 1 to 16 coils (NC2C waves of 8 coils, C2NC workgroups of 1, 2, 4
-and 8): every coil count at which the launch changes or leaves lanes idle, every kernel width with its own staging, several
-frames, samples per tile from none to several blocks and split tiles, each kind of
-dcw, and accumulation.
+and 8): every coil count at which the launch changes or leaves lanes idle, every
+kernel width with its own staging, several frames, samples per tile from none to
+several blocks and split tiles, each kind of dcw, and accumulation.
 
 Bar: relative L2 <= 1e-5 against the FP32 oracle, as the other 2D tests.
 """

@@ -162,3 +162,9 @@ def test_2d_c2nc_bad_cell_stays_in_its_windows(bad):
     assert inside.any() and not np.isfinite(b[3][inside]).any()
     assert np.array_equal(a[3][~near], b[3][~near])
     assert np.array_equal(np.delete(a, 3, 0), np.delete(b, 3, 0))
+
+
+@pytest.mark.parametrize("mode", [NFFT_conv_mode.NC2C, NFFT_conv_mode.C2NC])
+@pytest.mark.parametrize("C", [9, 16, 20, 33])
+def test_2d_windows_of_7_cells(C, mode):
+    assert max(errors(2, 64, 6.5, C, 4000, mode, True)) <= FP32
