@@ -52,11 +52,21 @@ def _stream():
 _PLANS = collections.OrderedDict()
 PLAN_CACHE_SIZE = 4
 
-# Plans that nothing uses any more, [(N, W, os_factor, device, stream), plan]: at
-# most PLAN_POOL_SIZE, given back by clear_plan_cache.  A deque's append and
-# popleft are atomic, so leases may end on any thread, in a collection too.
+# Plans that nothing uses any more, [(N, W, os_factor, device, stream), plan], the
+# longest unused first: at most PLAN_POOL_SIZE, the oldest dropped for a new one (so
+# that plans of sizes no longer in use give way), all given back by clear_plan_cache.
+# A deque's append and popleft are atomic, so leases may end on any thread, in a
+# collection too.
 _POOL = collections.deque()
 PLAN_POOL_SIZE = 2
+
+
+def _trim_pool():
+    while len(_POOL) > PLAN_POOL_SIZE:
+        try:
+            _POOL.popleft()
+        except IndexError:
+            return
 
 
 class _Lease:
@@ -69,23 +79,27 @@ class _Lease:
 
     def __del__(self):
         try:
-            if self.streams == {self.key[-1]} and len(_POOL) < PLAN_POOL_SIZE:
+            if self.streams == {self.key[-1]}:
                 _POOL.append((self.key, self.plan))
+                _trim_pool()
         except Exception:
             pass
 
 
 def _take(key):
-    """A pooled plan made with this key, or None."""
+    """A pooled plan made with this key, or None; the others keep their order."""
+    found = None
     for _ in range(len(_POOL)):
         try:
             entry = _POOL.popleft()
         except IndexError:
-            return None
-        if entry[0] == key:
-            return entry[1]
-        _POOL.append(entry)
-    return None
+            break
+        if found is None and entry[0] == key:
+            found = entry[1]
+        else:
+            _POOL.append(entry)
+    _trim_pool()  # leases may have ended meanwhile
+    return found
 
 
 def _plan_for(k, N, W, os_factor, stream):
