@@ -57,16 +57,15 @@ __device__ __forceinline__ TileSpan tile_span8(float p, const GridGeom& g, int d
 }
 
 // Positions, range flag and keys of the 2D hot path, one thread a sample.
-// raw: the caller's trajectory (null: pos holds the positions already).  wkeys /
-// wvals: the sample's tiles in `slots` slots, unused ones with the key past the
-// last (nkeys), which sorts behind every entry; hkeys / hvals: its home tile in
-// the C2NC binning gh.  Null arrays are left out.
+// raw: the caller's trajectory (null: pos holds the positions already).  wkeys: the
+// sample's tiles in `slots` slots, unused ones with the key past the last (nkeys),
+// which is no entry; hkeys / hvals: its home tile in the C2NC binning gh.  Null arrays
+// are left out.
 // Workgroup b takes samples [b chunk, (b + 1) chunk); wcnt / hcnt (or null) get its
 // entries of every key at [b nkeys + key] and [b nhome + key], counted in LDS.
 static __global__ __launch_bounds__(256) void prep2d_kernel(
     const float* __restrict__ raw, float* __restrict__ pos, long long nsamp, int chunk, long long M, GridGeom gw,
-    GridGeom gh, uint32_t nkeys, uint32_t nhome, int slots, uint32_t* __restrict__ wkeys, uint32_t* __restrict__ wvals,
-    uint32_t* __restrict__ hkeys, uint32_t* __restrict__ hvals, uint32_t* __restrict__ wcnt,
+    GridGeom gh, uint32_t nkeys, uint32_t nhome, int slots, uint32_t* __restrict__ wkeys, uint32_t* __restrict__ hkeys, uint32_t* __restrict__ hvals, uint32_t* __restrict__ wcnt,
     uint32_t* __restrict__ hcnt, int* __restrict__ flag) {
     extern __shared__ uint32_t counts[];
     uint32_t* wc = counts;
@@ -104,14 +103,10 @@ static __global__ __launch_bounds__(256) void prep2d_kernel(
                     if (a < sx.n && b < sy.n && o < slots) {
                         const uint32_t key = base + (uint32_t)(sx.t[a] + gw.ntiles[0] * sy.t[b]);
                         wkeys[j * slots + o] = key;
-                        if (wvals) wvals[j * slots + o] = (uint32_t)j;
                         if (wcnt) atomicAdd(&wc[key], 1u);
                         o++;
                     }
-            for (; o < slots; o++) {
-                wkeys[j * slots + o] = nkeys;
-                if (wvals) wvals[j * slots + o] = (uint32_t)j;
-            }
+            for (; o < slots; o++) wkeys[j * slots + o] = nkeys;
         }
         if (hkeys) {
             float pw;
@@ -316,7 +311,7 @@ __device__ __forceinline__ ItemSums block_exclusive(ItemSums v, ItemSums* sh, It
     return ItemSums{base.work + x.work - v.work, base.parts + x.parts - v.parts, base.items + x.items - v.items};
 }
 
-// One binning of items_kernel.
+// One binning of items_tables_kernel's work items.
 struct ItemArgs {
     const uint32_t* start;  // first entry of each key, nkeys + 1
     uint32_t nkeys;

@@ -8,6 +8,7 @@ bitwise repeatability over repeated preprocesses.
 """
 import numpy as np
 import pytest
+import torch
 
 from gadgetron_amd import DeviceArray, GTError, NFFT_prep_mode, NFFTPlan
 from gadgetron_amd import NFFT_comp_mode as CM
@@ -119,3 +120,34 @@ def test_sort_paths(F, M):
     op.preprocess(k1)
     assert rel_l2(ri, op.compute(smp, ri.shape, po.BACKWARDS_NC2C)) <= 1e-5
     assert rel_l2(rs, op.compute(img, rs.shape, po.FORWARDS_C2NC)) <= 1e-5
+
+
+def test_many_samples_with_short_last_tiles():
+    # 280,000 samples, past the counting sort, on a grid whose last tiles hold 2 cells: up to
+    # 9 tiles a window, 2.9 on average.  Results against the oracle, and the plan's memory:
+    # per sample 128 B of C2NC weights, 8 of positions and 4 of its list, 76 B of tables and
+    # list per entry: 360 B, below 450 with the grids and the allocations' granularity (9
+    # slots of tables and scratch a sample took over 900).
+    print("280,000 samples on 66 x 58", flush=True)
+    N, Nos, M = [44, 40], [66, 58], 280000
+    rng = np.random.default_rng(8)
+    k = rng.uniform(-0.5, 0.5, (1, M, 2)).astype(np.float32)
+    smp = (rng.standard_normal((1, 1, M)) + 1j * rng.standard_normal((1, 1, M))).astype(np.complex64)
+    img = (rng.standard_normal((1, 1, 40, 44)) + 1j * rng.standard_normal((1, 1, 40, 44))).astype(np.complex64)
+    warm = NFFTPlan(N, Nos, W=5.5)
+    warm.preprocess(DeviceArray.from_numpy(k))
+    plan = NFFTPlan(N, Nos, W=5.5)
+    d_k, d_s, d_x = (DeviceArray.from_numpy(a) for a in (k, smp, img))
+    oi, os_ = DeviceArray.zeros(img.shape, np.complex64), DeviceArray.zeros(smp.shape, np.complex64)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    plan.preprocess(d_k)
+    used = free - torch.cuda.mem_get_info()[0]
+    print(f"  {used / M:.0f} B a sample", flush=True)
+    assert used <= 450 * M
+    plan.compute(d_s, oi, None, CM.BACKWARDS_NC2C)
+    plan.compute(d_x, os_, None, CM.FORWARDS_C2NC)
+    op = po.Plan(N, 5.5, Nos=Nos, precision="float", cu=True)
+    op.preprocess(k)
+    assert rel_l2(oi.numpy(), op.compute(smp, img.shape, po.BACKWARDS_NC2C)) <= 1e-5
+    assert rel_l2(os_.numpy(), op.compute(img, smp.shape, po.FORWARDS_C2NC)) <= 1e-5
