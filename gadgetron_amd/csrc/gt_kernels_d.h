@@ -403,14 +403,16 @@ __global__ __launch_bounds__(256) void c2nc_split2d_d_kernel(const double2* __re
         cq[d] = cw;
     }
     const int iy = q & 7, x0 = (q >> 3) * XH;
-    const double wy = __shfl(wq[1], min(iy, KW - 1), 16) * (iy < KW ? 1.0 : 0.0);
+    const double wyq = __shfl(wq[1], min(iy, KW - 1), 16);
+    const double wy = iy < KW ? wyq : 0.0;
     const int cy = __shfl(cq[1], min(iy, KW - 1), 16);
     double wx[XH];
     int cx[XH];
 #pragma unroll
     for (int i = 0; i < XH; i++) {
         const int s = min(x0 + i, KW - 1);
-        wx[i] = x0 + i < KW ? __shfl(wq[0], s, 16) : __shfl(wq[0], s, 16) * 0.0;
+        const double w = __shfl(wq[0], s, 16);  // by every lane: the slot's lane has to take part
+        wx[i] = x0 + i < KW ? w : 0.0;
         cx[i] = __shfl(cq[0], s, 16);
     }
     const double2* row = grid + ((long long)f * g.G + (long long)g.nos[0] * cy);

@@ -1,7 +1,7 @@
 """Double-precision 2D gridding over 8 x 8 tiles (NC2C) and 16 lanes a sample
 (C2NC): grids whose last tile is short, small grids whose windows come back to
-their first tile, every window class (up to 8 cells, and 9 on the general
-kernels), coil counts around the register chunks, dense (split) and empty tiles.
+their first tile, every window class (windows of 9 cells gather with the general
+kernel), coil counts around the register chunks, dense (split) and empty tiles.
 
 Bar: relative L2 <= 1e-10 against the FP64 oracle, as the other double tests.
 """
@@ -16,7 +16,8 @@ from tests.helpers import rel_l2
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("Nos,W", [([12, 10], 5.5), ([16, 24], 2.5), ([34, 42], 5.5), ([46, 30], 7.5), ([50, 36], 8.5)])
+@pytest.mark.parametrize("Nos,W", [([12, 10], 5.5), ([16, 24], 2.5), ([34, 42], 5.5), ([46, 30], 7.5), ([50, 36], 8.5),
+                                   ([34, 42], 3.5), ([46, 30], 4.5), ([50, 36], 6.5)])
 @pytest.mark.parametrize("C", [1, 4, 5, 9])
 def test_double_2d(Nos, W, C):
     print(f"N_os {Nos}, W {W}, {C} coils", flush=True)
