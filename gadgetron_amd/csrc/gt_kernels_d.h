@@ -305,6 +305,7 @@ __global__ __launch_bounds__(64) void nc2c_cell2d_d_kernel(const double2* __rest
     for (int c = 0; c < CC; c++) acc[c] = make_double2(0.0, 0.0);
     for (uint32_t e0 = it.begin; e0 < it.end; e0 += kDChunk) {
         const uint32_t e = e0 + (uint32_t)lane;
+        double finite = 0.0;  // or NaN, with a sample that is not finite
         if (e < it.end) {
             const uint32_t j = tile_samples[e];
 #pragma unroll
@@ -317,6 +318,7 @@ __global__ __launch_bounds__(64) void nc2c_cell2d_d_kernel(const double2* __rest
                     s.x *= d;
                     s.y *= d;
                 }
+                finite += s.x * 0.0 + s.y * 0.0;
                 sm[c][lane] = s;
             }
 #pragma unroll
@@ -335,14 +337,21 @@ __global__ __launch_bounds__(64) void nc2c_cell2d_d_kernel(const double2* __rest
         }
         __syncthreads();
         const int n = (int)min((uint32_t)kDChunk, it.end - e0);
-#pragma unroll 2
-        for (int k = 0; k < n; k++) {
-            const double w = wt[0][k][lx] * wt[1][k][ly];
+        auto add = [&](int k, double w) {
 #pragma unroll
             for (int c = 0; c < CC; c++) {
                 const double2 s = sm[c][k];
                 acc[c].x += s.x * w;
                 acc[c].y += s.y * w;
+            }
+        };
+        if (__builtin_amdgcn_ballot_w64(finite != 0.0) == 0) {
+#pragma unroll 2
+            for (int k = 0; k < n; k++) add(k, wt[0][k][lx] * wt[1][k][ly]);
+        } else {  // an infinite or NaN sample stays in its window
+            for (int k = 0; k < n; k++) {
+                const double w = wt[0][k][lx] * wt[1][k][ly];
+                if (w != 0.0) add(k, w);
             }
         }
         __syncthreads();

@@ -8,7 +8,7 @@ Bar: relative L2 <= 1e-10 against the FP64 oracle, as the other double tests.
 import numpy as np
 import pytest
 
-from gadgetron_amd import DeviceArray, NFFTPlan
+from gadgetron_amd import DeviceArray, NFFT_conv_mode, NFFTPlan
 from gadgetron_amd import NFFT_comp_mode as CM
 from oracle import pyoracle as po
 from tests.helpers import rel_l2
@@ -42,3 +42,28 @@ def test_double_2d(Nos, W, C):
         e2 = rel_l2(os_.numpy(), op.compute(img, (C, F, M), po.FORWARDS_C2NC, dcw=dcw))
         print(f"  adjoint {e1:.2e}, forward {e2:.2e}", flush=True)
         assert e1 <= 1e-10 and e2 <= 1e-10
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_bad_sample_stays_in_its_window(bad):
+    print(f"double 2D 64^2, 5 coils, one sample {bad}", flush=True)
+    rng = np.random.default_rng(1)
+    nos, C, W, M, j = 96, 5, 5.5, 3000, 11
+    k = rng.uniform(-0.5, 0.5, (1, M, 2))
+    plan = NFFTPlan([64, 64], None, W=W, os_factor=1.5, precision="double")
+    plan.preprocess(DeviceArray.from_numpy(k))
+    x = rng.standard_normal((C, 1, M)) + 1j * rng.standard_normal((C, 1, M))
+    y = x.copy()
+    y[3, 0, j] = bad
+    outs = []
+    for s in (x, y):
+        out = DeviceArray.zeros((C, 1, nos, nos), np.complex128)
+        plan.convolve(DeviceArray.from_numpy(s), out, NFFT_conv_mode.NC2C)
+        outs.append(out.numpy()[:, 0])
+    a, b = outs
+    hit = np.zeros((nos, nos), bool)
+    win = [np.arange(np.ceil(p - W / 2), np.floor(p + W / 2) + 1).astype(int) % nos for p in (k[0, j] + 0.5) * nos]
+    hit[np.ix_(win[1], win[0])] = True
+    assert not np.isfinite(b[3][hit]).any()
+    assert np.array_equal(a[3][~hit], b[3][~hit])
+    assert np.array_equal(np.delete(a, 3, 0), np.delete(b, 3, 0))
