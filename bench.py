@@ -247,7 +247,7 @@ def batched_cgsense(nprob=64, iterations=10, reps=3, seed=3):
         "rel_err_graph_branches_vs_plain": rel_to_plain(xb),
         "rel_err_fused_vs_plain": rel_to_plain(xf),
         "note": "plain: the reference's per-problem loop (dot products read back each iteration); "
-                "graph_branches: each problem's whole solve in one hipGraph, problems on parallel branches; "
+                "graph_branches: every problem's whole solve in one hipGraph, one after the other; "
                 "fused: one launch per step for all 64 problems (descriptor tables), captured in one hipGraph",
     }
 

@@ -23,7 +23,6 @@
 #include <map>
 #include <memory>
 #include <mutex>
-#include <numeric>
 #include <string>
 #include <utility>
 #include <vector>
@@ -902,13 +901,12 @@ struct gt_cg_batch {
     int device = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    int branches = 0;  // chosen by tune_graph
+    int branches = 0;  // of the recorded graph (GT_CG_BATCHED: one chain)
     // generations of each problem's plan and operator when the graph was
     // recorded: a replay after either changed would use stale addresses and
     // launch sizes
     std::vector<std::pair<uint64_t, uint64_t>> gens;
-    std::vector<hipStream_t> streams;
-    std::vector<hipEvent_t> events;
+    hipStream_t stream = nullptr;  // the graphs are recorded on it
     // GT_CG_FUSED: the fused gridding of every problem, the CG vectors (r, p,
     // q, mhd of every problem in one allocation), states and partial sums,
     // and the per-problem table the batched CG kernels read
@@ -918,99 +916,42 @@ struct gt_cg_batch {
     ~gt_cg_batch() {
         if (exec) (void)hipGraphExecDestroy(exec);
         if (graph) (void)hipGraphDestroy(graph);
-        for (auto e : events) (void)hipEventDestroy(e);
-        for (auto s : streams) (void)hipStreamDestroy(s);
+        if (stream) (void)hipStreamDestroy(stream);
         if (fused) fused_destroy(fused);
     }
 };
 
 namespace {
 
-// Problems longest first onto the least loaded branch.  Cost of a solve ~
-// samples x coils + grid x coils (bandwidth) plus a fixed term for its ~150
-// launches (small problems are latency bound).
-std::vector<std::vector<int>> assign_branches(const std::vector<gt_sense_op*>& ops, int nbr) {
-    std::vector<int> order(ops.size());
-    std::iota(order.begin(), order.end(), 0);
-    auto work = [&](int i) {
-        const gt_sense_op* o = ops[size_t(i)];
-        return double(o->M * o->F * o->C) + 2.25 * double(o->nimg * o->F * o->C) + 4.0e5;
-    };
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return work(a) > work(b); });
-    std::vector<std::vector<int>> br(static_cast<size_t>(nbr));
-    std::vector<double> load(static_cast<size_t>(nbr), 0.0);
-    for (int i : order) {
-        const size_t k = size_t(std::min_element(load.begin(), load.end()) - load.begin());
-        br[k].push_back(i);
-        load[k] += work(i);
-    }
-    return br;
+// Records fn's launches as one chain into b->graph / b->exec, on a stream of
+// its own (the caller's may be the null stream, which cannot be captured).  The
+// instantiated graph is launched on the caller's stream.
+template <typename Fn>
+void record_graph(gt_cg_batch* b, Fn&& fn) {
+    if (!b->stream) GT_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
+    if (b->exec) (void)hipGraphExecDestroy(b->exec);
+    if (b->graph) (void)hipGraphDestroy(b->graph);
+    b->exec = nullptr;
+    b->graph = nullptr;
+    GT_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
+    fn(b->stream);
+    GT_HIP(hipStreamEndCapture(b->stream, &b->graph));
+    GT_HIP(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
 }
 
-// Captures one graph with nbr parallel branches, on a stream of its own (the
-// caller's may be the null stream, which cannot be captured): fork from the
-// capture stream, each branch runs its problems' whole solves back to back,
-// join.  The instantiated graph is launched on the caller's stream.
-void build_graph(gt_cg_batch* b, int nbr, hipGraph_t* graph, hipGraphExec_t* exec) {
-    auto br = assign_branches(b->ops, nbr);
-    while (int(b->streams.size()) < nbr + 1) {
-        hipStream_t st;
-        GT_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-        b->streams.push_back(st);
-    }
-    while (int(b->events.size()) < nbr + 1) {
-        hipEvent_t e;
-        GT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        b->events.push_back(e);
-    }
-    hipStream_t s = b->streams[size_t(nbr)];
-    GT_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    GT_HIP(hipEventRecord(b->events[0], s));
-    for (int k = 0; k < nbr; k++) {
-        hipStream_t bs = b->streams[size_t(k)];
-        GT_HIP(hipStreamWaitEvent(bs, b->events[0], 0));
-        for (int i : br[size_t(k)]) cg_solve(b->ops[size_t(i)], b->data[size_t(i)], b->x[size_t(i)], &b->desc, false, bs);
-        GT_HIP(hipEventRecord(b->events[size_t(k) + 1], bs));
-        GT_HIP(hipStreamWaitEvent(s, b->events[size_t(k) + 1], 0));
-    }
-    GT_HIP(hipStreamEndCapture(s, graph));
-    GT_HIP(hipGraphInstantiate(exec, *graph, nullptr, nullptr, 0));
-}
-
-// Autotuner: the number of parallel branches that runs the batch fastest.
-// Each candidate graph is built and replayed twice (the second replay timed on
-// the host around a synchronisation); the fastest is kept.
-void tune_graph(gt_cg_batch* b, hipStream_t s) {
-    const int n = int(b->ops.size());
-    std::vector<int> cand;
-    for (int c : {2, 4, 8, 16, 32, 64})
-        if (c < n) cand.push_back(c);
-    cand.push_back(n);  // one branch per problem
-    if (cand.empty()) cand.push_back(1);
-    double best = 1e300;
-    for (int nbr : cand) {
-        hipGraph_t g = nullptr;
-        hipGraphExec_t e = nullptr;
-        build_graph(b, nbr, &g, &e);
-        GT_HIP(hipGraphLaunch(e, s));
-        GT_HIP(hipStreamSynchronize(s));
-        const auto t0 = std::chrono::steady_clock::now();
-        GT_HIP(hipGraphLaunch(e, s));
-        GT_HIP(hipGraphLaunch(e, s));
-        GT_HIP(hipStreamSynchronize(s));
-        const double t = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-        if (t < best) {
-            best = t;
-            if (b->exec) (void)hipGraphExecDestroy(b->exec);
-            if (b->graph) (void)hipGraphDestroy(b->graph);
-            b->graph = g;
-            b->exec = e;
-            b->branches = nbr;
-        } else {
-            (void)hipGraphExecDestroy(e);
-            (void)hipGraphDestroy(g);
-        }
-    }
+// GT_CG_BATCHED: the problems' whole solves one after the other.  Parallel
+// branches (problems spread over forked capture streams, up to one branch per
+// problem) ran the 64 problems of the uneven workload in 34 ms, a chain takes
+// 63; they are off because creating such a graph once ended the host
+// process with a segmentation fault whose cause is not known.
+// One replay here, so that the caller's first run is as long as the next.
+void batched_setup(gt_cg_batch* b, hipStream_t s) {
+    record_graph(b, [&](hipStream_t cs) {
+        for (size_t i = 0; i < b->ops.size(); i++) cg_solve(b->ops[i], b->data[i], b->x[i], &b->desc, false, cs);
+    });
+    b->branches = 1;
+    GT_HIP(hipGraphLaunch(b->exec, s));
+    GT_HIP(hipStreamSynchronize(s));
 }
 
 // GT_CG_FUSED: the whole batch's solve, one launch per step for every problem
@@ -1076,21 +1017,7 @@ void fused_setup(gt_cg_batch* b, hipStream_t s) {
     b->fprobs.reserve(size_t(n) * sizeof(CgProb));
     GT_HIP(hipMemcpyAsync(b->fprobs.ptr, probs.data(), size_t(n) * sizeof(CgProb), hipMemcpyHostToDevice, s));
     GT_HIP(hipStreamSynchronize(s));
-    // record the solve on a stream of its own (the caller's may be the null stream)
-    if (b->streams.empty()) {
-        hipStream_t st;
-        GT_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-        b->streams.push_back(st);
-    }
-    hipStream_t cs = b->streams[0];
-    if (b->exec) (void)hipGraphExecDestroy(b->exec);
-    if (b->graph) (void)hipGraphDestroy(b->graph);
-    b->exec = nullptr;
-    b->graph = nullptr;
-    GT_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-    fused_solve(b, cs);
-    GT_HIP(hipStreamEndCapture(cs, &b->graph));
-    GT_HIP(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
+    record_graph(b, [&](hipStream_t cs) { fused_solve(b, cs); });
 }
 
 // Autotuner of the fused batch: NC2C table entries per work item, applied to
@@ -1322,7 +1249,7 @@ gt_status gt_cgsense_batch_create(gt_cg_batch** out, gt_sense_op* const* ops, co
             GT_REQUIRE(ops[i] && data[i] && x[i], GT_ERR_INVALID_ARGUMENT, "null problem entry");
             for (int j = 0; j < i; j++)
                 GT_REQUIRE(ops[j] != ops[i] && ops[j]->plan != ops[i]->plan, GT_ERR_INVALID_ARGUMENT,
-                           "problems of one batch need their own operator and plan (the branches run concurrently)");
+                           "problems of one batch need their own operator and plan");
             validate_sizes(ops[i], desc);
             ops[i]->reserve_cg(desc->iterations, desc->n_regs > 0);
             ops[i]->warm(s);
@@ -1330,7 +1257,7 @@ gt_status gt_cgsense_batch_create(gt_cg_batch** out, gt_sense_op* const* ops, co
             b->data.push_back(data[i]);
             b->x.push_back(x[i]);
         }
-        if (mode == GT_CG_BATCHED) tune_graph(b.get(), s);
+        if (mode == GT_CG_BATCHED) batched_setup(b.get(), s);
         if (mode == GT_CG_FUSED) fused_tune(b.get(), s);
         if (mode != GT_CG_PLAIN)
             for (auto* o : b->ops) b->gens.emplace_back(plan_generation(o->plan), o->generation);

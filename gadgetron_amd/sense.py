@@ -107,7 +107,7 @@ class CgBatch:
 
     mode "plain": one problem at a time with the dot products read back to the
     host each time (the reference's method); "batched": every solve captured
-    into one hipGraph with the problems on parallel branches; "fused": one
+    into one hipGraph, one problem after the other; "fused": one
     launch per step for every problem (gridding over all problems' work items,
     FFT passes per size group, CG updates with a problem index), captured into
     one hipGraph (2D plans, identity regulariser only)."""
@@ -134,7 +134,7 @@ class CgBatch:
 
     @property
     def branches(self):
-        """Parallel graph branches the autotuner chose (0 for the plain mode)."""
+        """Branches of the recorded graph (1 for "batched", 0 for the other modes)."""
         n = ctypes.c_int()
         check(lib().gt_cgsense_batch_branches(self._h, ctypes.byref(n)))
         return n.value

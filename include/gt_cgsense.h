@@ -99,9 +99,8 @@ gt_status gt_cgsense_solve_image(gt_sense_op* op, const void* rhs, void* x, cons
  *   GT_CG_PLAIN:   one problem at a time, each iteration's dot products read
  *                  back to the host, as the reference's cgSolver does;
  *   GT_CG_BATCHED: every problem's whole solve (all iterations) captured into
- *                  one hipGraph with the problems spread over parallel
- *                  branches (longest first), launched as one graph with no
- *                  host round trips;
+ *                  one hipGraph, one problem after the other, launched as one
+ *                  graph with no host round trips;
  *   GT_CG_FUSED:   every step of every problem in one launch, from
  *                  per-problem descriptor tables: one gridding launch per
  *                  direction over the work items of all problems, the FFT
@@ -116,9 +115,9 @@ gt_status gt_cgsense_solve_image(gt_sense_op* op, const void* rhs, void* x, cons
  * choose by coil count), so its results agree with theirs to rounding. */
 enum { GT_CG_PLAIN = 0, GT_CG_BATCHED = 1, GT_CG_FUSED = 2 };
 typedef struct gt_cg_batch gt_cg_batch;
-/* gt_cgsense_batch_create (GT_CG_BATCHED) times candidate graphs by running
- * them: it writes every problem's x (whole solves), reads the data and runs
- * one E^H E per operator to size its workspaces.  After creation the caller
+/* gt_cgsense_batch_create (GT_CG_BATCHED) runs its graph once: it writes every
+ * problem's x (whole solves), reads the data and runs one E^H E per operator to
+ * size its workspaces.  After creation the caller
  * may change the contents of data (and x, which each run overwrites) but not
  * the bound plans (no preprocess or set_tiling) nor the operators' sizes:
  * gt_cgsense_batch_run then returns GT_ERR_INVALID_ARGUMENT without running
@@ -128,8 +127,8 @@ gt_status gt_cgsense_batch_create(gt_cg_batch** batch, gt_sense_op* const* ops, 
                                   void* const* x, int nprob, const gt_cg_desc* desc, int mode, gt_stream_t stream);
 gt_status gt_cgsense_batch_run(gt_cg_batch* batch, gt_stream_t stream);
 gt_status gt_cgsense_batch_destroy(gt_cg_batch* batch);
-/* Parallel branches of a batched graph, picked at creation by timing one
- * replay per candidate (2, 4, ..., 64, and one per problem); 0 for GT_CG_PLAIN. */
+/* Parallel branches of a batched graph: 1 for GT_CG_BATCHED (one chain), 0 for
+ * the other modes. */
 gt_status gt_cgsense_batch_branches(const gt_cg_batch* batch, int* branches);
 /* GT_CG_FUSED: NC2C table entries per work item its autotuner chose for every
  * bound plan (0: each plan's own rule; -1 for the other modes).  Creation tries
