@@ -124,7 +124,7 @@ def cpu_baseline(wl, samples, budget_s):
 
 
 # the gridding runs on the matrix cores unless GT_NUFFT_MFMA=0; 2D: the kernels of the 32-coil
-# workloads (NC2C of up to 8 coils: nc2c_mfma2d8_kernel, C2NC of up to 16: c2nc_mfma2d16_kernel)
+# workloads (NC2C of up to 8 coils: nc2c_mfma2d8_kernel, C2NC of up to 16: c2nc_gather2d_kernel)
 _FP32_GRIDDING = os.environ.get("GT_NUFFT_MFMA", "1").startswith("0")
 KERNELS_2D = {"nc2c": ("nc2c_reg2d_kernel" if _FP32_GRIDDING else "nc2c_mfma2d_kernel") + " + nc2c_reduce2d_kernel",
               "c2nc": "c2nc_multi2d_kernel" if _FP32_GRIDDING else "c2nc_mfma2d_kernel"}

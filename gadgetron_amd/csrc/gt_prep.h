@@ -14,8 +14,11 @@
 // 84 with items and tables in one launch (items_tables_kernel).  Preprocess alone,
 // sorted by the library / by counting / in one launch with the tables, us: 13 k
 // samples on 288^2 124 / 66 / 54, 66 k on 384^2 201 / 85 / 69, 262 k 378 / 165 / 130,
-// 66 k on 768^2 216 / 175 / 116, 262 k 370 / 266 / 176; past the bounds the library's
-// radix passes have enough work.
+// 66 k on 768^2 216 / 175 / 116, 262 k 370 / 266 / 176.  Past the bounds the library's
+// radix passes have enough work; there the entries are counted first, with a read-back
+// more, so that the tables have their size and not that of the most tiles a window can
+// touch (922 k samples on 512^2: 308 MB a plan against 516; 410 k on 768^2: 0.92 ms
+// against 0.67).
 #pragma once
 
 #include <hip/hip_runtime.h>
